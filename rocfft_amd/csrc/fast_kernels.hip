@@ -268,10 +268,6 @@ extern "C" const FastEntry* FAST_SLICE_FN(FAST_SLICE)(int* count)
 }
 
 #if FAST_SLICE == 0
-#define FAST_SLICE_LIST(X)                                                                              \
-    X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16) X(17) X(18) \
-        X(19) X(20) X(21) X(22) X(23)
-static_assert(FAST_SLICES == 24, "FAST_SLICE_LIST names twenty-four slices");
 #define FAST_DECLARE(I) extern "C" const FastEntry* fftrt_fast_slice_##I(int*);
 FAST_SLICE_LIST(FAST_DECLARE)
 

@@ -523,13 +523,14 @@ static rocfft_status execute_impl(const rocfft_plan plan, void* in_buffer[], voi
         // the work area of the pass list these buffers get (staged copies are aligned allocations)
         size_t need = staging ? ep.work_bytes()
                               : select_exec_plan(ep, in, out, work_hint, fused ? &ecb : nullptr).own_work_bytes();
-        // A list with tall columns needs less than the same plan without them.  What an area that is
-        // not allocated here has to hold is the latter all the same, so that the areas accepted do
-        // not depend on the kernels that run.
-        size_t room = need;
-        for(const PassRec& r : ep.passes)
-            if(!staging && r.kind == PASS_TALL && ep.unaligned)
-                room = std::max(room, select_exec_plan(*ep.unaligned, in, out, work_hint, fused ? &ecb : nullptr).own_work_bytes());
+        // A list with tall columns needs less than the same plan without them.  Whether a call is
+        // accepted goes by the latter all the same (an area given or the static one has to hold it,
+        // and where neither is there the stream must not be capturing), so that it does not depend on
+        // the kernels that run; an area allocated here is as large as the list needs.
+        const size_t room
+            = ep.tall && !staging
+                  ? std::max(need, select_exec_plan(*ep.unaligned, in, out, work_hint, fused ? &ecb : nullptr).own_work_bytes())
+                  : need;
         void* work = nullptr;
         bool  own  = false;
         if(room && static_work)
@@ -552,15 +553,15 @@ static rocfft_status execute_impl(const rocfft_plan plan, void* in_buffer[], voi
                     return rocfft_status_invalid_work_buffer;
                 work = info->workBuffer;
             }
-            else if(!staging && need)
+            else if(!staging)
             {
                 // no caller-owned scratch: allocate for this call (reference
                 // transform.cpp:424-434); impossible while the stream is being captured
                 if(fftrt_stream_capturing(stream))
                     return rocfft_status_invalid_work_buffer;
-                if(fftrt_malloc(&work, need) != 0)
+                if(need && fftrt_malloc(&work, need) != 0)
                     return rocfft_status_failure;
-                own = true;
+                own = need != 0;
             }
         }
         if(pass_ms && fftrt_stream_capturing(stream))

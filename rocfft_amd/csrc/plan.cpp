@@ -3141,6 +3141,7 @@ rocfft_status build_exec_plan(const Problem& p, ExecPlan& plan, bool dry, std::s
         if(build_exec_plan(p, *alt, dry, alt_err, half_io) == rocfft_status_success)
         {
             plan.unaligned = alt;
+            plan.tall      = true;
             return st;
         }
         // (callbacks and such buffers have to be accepted: without that list, this plan is not used)

@@ -108,6 +108,7 @@ struct ExecPlan
     // executor when a buffer fails the alignment test (the reference accepts such buffers).
     // The second list of a plan with tall column passes is the plan made without them.
     std::shared_ptr<ExecPlan> unaligned;
+    bool                      tall = false; // has tall column passes (then there is a second list)
     size_t                    own_work_bytes() const
     {
         return (tmp_elems + blu_elems + cpx_elems) * elem_bytes;

@@ -11,6 +11,9 @@
 #include "gpu_rt.h"
 #include "fast_core.h"
 #include "tile_core.h"
+#include <algorithm>
+#include <cmath>
+#include <complex>
 #include <cstdlib>
 #include <cstring>
 #include <vector>
@@ -94,6 +97,87 @@ void emu_tile(const fftk_params& p, uint32_t grid, size_t lds_bytes)
 }
 } // namespace
 
+// The tall column kernel: the schedules of the real one, so that the planner makes the same plans, and
+// for each column of a tile a plain mixed-radix transform on what the kernel's parameters say.
+namespace
+{
+struct EmuTall
+{
+    uint32_t n;
+    int      precision;
+    uint32_t radix[4], tpt, width, threads, pitch;
+};
+#define TALL_SCHED(SLICE, T, N, A, B, C, D, TPT, W, SHIFT) \
+    {N, sizeof(T) == sizeof(double) ? 1 : 0, {A, B, C, D}, TPT, W, (TPT * W + 63) / 64 * 64, N + ((N - 1) >> SHIFT)},
+const EmuTall g_tall[] = {
+#include "tall_schedules.h"
+};
+#undef TALL_SCHED
+
+const EmuTall* emu_tall(int precision, uint32_t n)
+{
+    for(const EmuTall& e : g_tall)
+        if(e.n == n && e.precision == precision)
+            return &e;
+    return nullptr;
+}
+
+typedef std::complex<double> Z;
+void emu_dft(const Z* in, size_t stride, Z* out, uint32_t n, const uint32_t* radix, int dir)
+{
+    if(n == 1)
+    {
+        out[0] = in[0];
+        return;
+    }
+    const uint32_t r = radix[0], m = n / r;
+    std::vector<Z> part(n);
+    for(uint32_t a = 0; a < r; ++a)
+        emu_dft(in + a * stride, stride * r, part.data() + a * m, m, radix + 1, dir);
+    for(uint32_t k = 0; k < n; ++k)
+    {
+        Z sum = 0;
+        for(uint32_t a = 0; a < r; ++a)
+            sum += part[a * m + k % m] * std::polar(1.0, dir * 2 * M_PI * ((uint64_t)a * k % n) / n);
+        out[k] = sum;
+    }
+}
+
+template <typename T>
+void emu_tall_run(const fftk_params& p)
+{
+    typedef typename cplx_of<T>::type C;
+    for(uint32_t bid = 0; bid < p.grid; ++bid)
+    {
+        TileCtx<T> c;
+        tile_decode<T>(p, bid, c);
+        const C* src = reinterpret_cast<const C*>(static_cast<const T*>(p.in0) + c.ibase);
+        C*       dst = reinterpret_cast<C*>(static_cast<T*>(p.out0) + c.obase);
+        const uint32_t cols = std::min(p.W, p.tile_cnt - c.tile0);
+        std::vector<Z> x((size_t)cols * p.n), y(p.n);
+        // every load of a tile comes before its first store
+        for(uint32_t w = 0; w < cols; ++w)
+            for(uint32_t j = 0; j < p.n; ++j)
+            {
+                const C v              = src[(uint64_t)j * p.t_is_c + w];
+                x[(size_t)w * p.n + j] = Z(v.x, v.y);
+            }
+        for(uint32_t w = 0; w < cols; ++w)
+        {
+            emu_dft(&x[(size_t)w * p.n], 1, y.data(), p.n, p.radix, p.dir);
+            const double scale = (p.flags & FFTK_F_SCALE) ? p.scale : 1;
+            for(uint32_t k = 0; k < p.n; ++k)
+            {
+                C v;
+                v.x = (T)(y[k].real() * scale);
+                v.y = (T)(y[k].imag() * scale);
+                dst[(uint64_t)k * p.t_os_c + w] = v;
+            }
+        }
+    }
+}
+} // namespace
+
 extern "C" {
 
 int fftrt_device_count(int* count)
@@ -151,9 +235,15 @@ int fftrt_device_sync(void)
 {
     return 0;
 }
+// (tests) what the next calls are told about their stream
+static int g_capturing = 0;
+__attribute__((visibility("default"))) void fftrt_emu_set_capturing(int on)
+{
+    g_capturing = on;
+}
 int fftrt_stream_capturing(void*)
 {
-    return 0;
+    return g_capturing;
 }
 
 // The emulation only has the generic kernel, but it reports the pass schedules of the
@@ -282,14 +372,43 @@ int fftrt_launch_fast2d_real(const struct fftk_params*, int, int, uint32_t, size
     return 1;
 }
 
-// no tall column kernel in the emulation: such dimensions take the tile passes here
-int fftrt_tall_info(int, uint32_t, uint32_t*, uint32_t*, uint32_t*, uint32_t*, uint32_t*, uint32_t*)
+static int g_tall_on = 0;
+// (tests) whether plans made from here on may have tall column passes; off unless a test asks
+__attribute__((visibility("default"))) void fftrt_emu_set_tall(int on)
 {
-    return 0;
+    g_tall_on = on;
 }
-int fftrt_launch_tall(const struct fftk_params*, int, void*)
+int fftrt_tall_info(int precision, uint32_t n, uint32_t* radix, uint32_t* nf, uint32_t* tpt, uint32_t* width,
+                    uint32_t* threads, uint32_t* pitch)
 {
+    const EmuTall* e = g_tall_on ? emu_tall(precision, n) : nullptr;
+    if(!e)
+        return 0;
+    *nf = 0;
+    for(uint32_t r : e->radix)
+        if(r > 1)
+            radix[(*nf)++] = r;
+    *tpt     = e->tpt;
+    *width   = e->width;
+    *threads = e->threads;
+    *pitch   = e->pitch;
     return 1;
+}
+static long g_tall_launches = 0;
+// (tests) launches of the tall column kernel so far
+__attribute__((visibility("default"))) long fftrt_emu_tall_launches(void)
+{
+    return g_tall_launches;
+}
+int fftrt_launch_tall(const struct fftk_params* p, int precision, void*)
+{
+    const EmuTall* e = emu_tall(precision, p->n);
+    if(!e || p->T != e->tpt || p->nthreads != e->threads || p->W != e->width || p->pitch != e->pitch || p->w_inner
+       || p->grid != (p->tile_cnt + p->W - 1) / p->W * p->oc[0] * p->oc[1] * p->oc[2])
+        return 1;
+    ++g_tall_launches;
+    precision ? emu_tall_run<double>(*p) : emu_tall_run<float>(*p);
+    return 0;
 }
 
 int fftrt_has_big32k(void)

@@ -1352,7 +1352,8 @@ static TablePtr bluestein_spectrum(Builder& b, uint64_t N, uint64_t M, uint64_t 
                                    bool conj_chirp, uint64_t M2 = 1);
 static bool     big_eligible(const Builder& b, uint64_t n, int64_t t_is, int64_t t_os,
                              const std::vector<Other>& others, const IoRef& src, const IoRef& dst);
-static uint32_t tall_width(uint64_t n, size_t esize, int64_t is, int64_t os);
+static bool     plan_tall(const Builder& b, uint64_t n, int64_t t_is, int64_t t_os, const std::vector<Other>& others,
+                          const IoRef& src, const IoRef& dst, int dir, double scale, bool has_scale, PassRec& rec);
 static bool     emit_tall(Builder& b, uint64_t n, int64_t t_is, int64_t t_os, const std::vector<Other>& others,
                           const IoRef& src, const IoRef& dst, int dir, double scale, bool has_scale);
 static void     emit_big(Builder& b, uint32_t mode, const std::vector<Other>& others, const IoRef& src,
@@ -2314,28 +2315,68 @@ static uint32_t tall_width(uint64_t n, size_t esize, int64_t is, int64_t os)
     // 3072 x 3840 x 3 364 -> 343 us, but rows of 64 KB 8192 x 4096 x 2 620 -> 667 us; up to 3500 points
     // also closer rows lose (15 KB, 1920 x 3072 x 4: 238 -> 247 us).  Double precision: rows of 48 KB
     // and more 4096 x 4096 x 2 625 -> 585 us, 3072 x 3072 x 2 356 -> 335 us, 8192 x 4096 652 -> 635 us; rows
-    // of 32 KB 2048 x 2560 x 2 193 -> 149 us, but 2048 x 4096 x 2 299 -> 307 us.
+    // of 32 KB 2048 x 2560 x 2 193 -> 149 us, but 2048 x 4096 x 2 299 -> 307 us; 2401 points lose from rows of
+    // 32 KB on (4096 columns 127 -> 148 us).
     const int64_t scalar = (int64_t)esize / 2;
     for(int64_t st : {is * scalar, os * scalar})
     {
         if(width * esize >= 64 || st % 512)
             continue;
-        if(esize == 8 ? (n <= 3500 || st > 32768) : (n > 3072 && st > 16384 && st < 49152))
+        if(esize == 8 ? (n <= 3500 || st > 32768) : (n > 3072 ? st > 16384 && st < 49152 : n < 2420 && st >= 32768))
             return 0;
     }
     return width;
 }
 
-// One strided dimension as a pass of the tall column kernel; false (nothing emitted) when the
+// Does one pass of the tall column kernel, `grid` workgroups over rows of `columns` columns, take less
+// time than the passes it would replace?  Measured with all its lengths, 4 to 20000 columns and rows of
+// 5 to 2000 columns in batches (1 to 7500 workgroups), both precisions.
+static bool tall_pays(uint64_t n, size_t esize, int64_t is, int64_t os, uint32_t width, uint32_t nf, uint32_t columns,
+                      uint64_t grid)
+{
+    if(getenv("ROCFFT_AMD_TALL_ANY_GRID")) // (tests of that kernel at small sizes)
+        return true;
+    // Idle columns in the last tile of a row, where a tile pass folds the batch into its tile axis:
+    // single precision 880 points, 9 columns x 40 11.9 against 14.7 us, 33 x 16 13.3 against 15.3 us.
+    const uint64_t tiles = ((uint64_t)columns + width - 1) / width;
+    if((uint64_t)columns * 20 < tiles * width * 17)
+        return false;
+    // One workgroup transforms twice the columns of a tile pass and many times those of a split, so a grid
+    // that leaves most compute units idle, or a last round that does, costs more than is won in memory:
+    // 64 columns of 2187 points 9.0 against 15.7 us, 16 of 3888 in double precision 9.3 against 17.7 us.
+    const uint64_t rounds = (grid + 255) / 256;
+    const bool     narrow = width * esize < 64;
+    const bool     one    = plain_dim_is_single(n, true, esize, is, os);
+    const int64_t  line   = 256 / (int64_t)esize; // scalars in 128 bytes
+    if(narrow || one)
+    {
+        // In the place of one tile pass, and with 32-byte runs, the gain is 5 to 20 %: all compute units but
+        // for an eighth in every round (3840 points in double precision: 256 columns, half a round, 18.5 against
+        // 22.8 us; 768, one and a half, 43.3 against 48.0 us; but 512, one, 30.8 against 27.9 us with this kernel).
+        // 32-byte runs in the place of one pass need rows that start on a 128-byte line (3000 points x 1000 columns
+        // 64.3 -> 39.0 us, but 2640 x 3001 104 -> 112 us).
+        if(narrow && one && (is % line || os % line))
+            return false;
+        return grid * 8 >= rounds * 256 * 7;
+    }
+    // In the place of two passes, single precision: from a quarter of a round on (1080 points x 512 columns the
+    // same 10.5 us either way, x 768 12.8 -> 10.9 us), with four radix passes three quarters (2025 x 1024, half a
+    // round, 20.3 against 23.2 us; x 1536 29.7 -> 25.2 us), and no last round mostly idle (1500 x 2560, one and a
+    // quarter, 33.4 against 36.1 us).
+    if(rounds == 1)
+        return grid >= (nf > 3 ? 192 : 65);
+    return grid * 5 >= rounds * 256 * 4;
+}
+
+// One strided dimension as a pass of the tall column kernel, without its tables; false when the
 // layout does not suit it: interleaved arrays, whole tiles of neighbouring columns on both sides,
 // 32-bit offsets inside a tile.
-static bool emit_tall(Builder& b, uint64_t n, int64_t t_is, int64_t t_os, const std::vector<Other>& others,
-                      const IoRef& src, const IoRef& dst, int dir, double scale, bool has_scale)
+static bool plan_tall(const Builder& b, uint64_t n, int64_t t_is, int64_t t_os, const std::vector<Other>& others,
+                      const IoRef& src, const IoRef& dst, int dir, double scale, bool has_scale, PassRec& rec)
 {
     uint32_t width = tall_width(n, b.esize, t_is, t_os);
     if(width == 0 || src.planar || dst.planar || src.im_delta != 1 || dst.im_delta != 1)
         return false;
-    PassRec rec;
     try
     {
         TileSpec s;
@@ -2371,16 +2412,11 @@ static bool emit_tall(Builder& b, uint64_t n, int64_t t_is, int64_t t_os, const 
     if(!fftrt_tall_info(b.precision, (uint32_t)n, radix, &nf, &tpt, &width, &threads, &pitch))
         return false;
     const uint64_t grid = (uint64_t)((k.tile_cnt + width - 1) / width) * k.oc[0] * k.oc[1] * k.oc[2];
-    if(grid == 0 || grid >= (1ull << 31))
+    if(grid == 0 || grid >= (1ull << 31) || !tall_pays(n, b.esize, t_is, t_os, width, nf, k.tile_cnt, grid))
         return false;
-    std::vector<uint32_t> schedule(radix, radix + nf);
-    uint32_t              twoff[FFTK_MAX_PASSES];
-    TablePtr              tw = stacked_twiddles(schedule, b.precision, b.dry, twoff);
     rec.tables.clear();
-    rec.tables.push_back(tw);
-    rec.kind   = PASS_TALL;
-    k.tw       = tw->dptr;
-    k.nf       = nf;
+    rec.kind = PASS_TALL;
+    k.nf     = nf;
     for(uint32_t i = 0; i < nf; ++i)
         k.radix[i] = radix[i];
     k.T        = tpt;
@@ -2390,8 +2426,21 @@ static bool emit_tall(Builder& b, uint64_t n, int64_t t_is, int64_t t_os, const 
     k.pitch    = pitch;
     rec.lds    = (size_t)pitch * width * b.esize;
     rec.grid = k.grid = (uint32_t)grid;
-    // neighbouring tiles share 128-byte lines unless tiles are whole lines of line-aligned rows
-    k.xcd_remap = (g_xcd_remap && grid >= 64 && (width < 16 || k.t_is % 32 || k.t_os % 32)) ? 1 : 0;
+    // neighbouring tiles share 128-byte lines
+    k.xcd_remap = (g_xcd_remap && grid >= 64) ? 1 : 0;
+    return true;
+}
+
+static bool emit_tall(Builder& b, uint64_t n, int64_t t_is, int64_t t_os, const std::vector<Other>& others,
+                      const IoRef& src, const IoRef& dst, int dir, double scale, bool has_scale)
+{
+    PassRec rec;
+    if(!plan_tall(b, n, t_is, t_os, others, src, dst, dir, scale, has_scale, rec))
+        return false;
+    uint32_t twoff[FFTK_MAX_PASSES];
+    TablePtr tw = stacked_twiddles(std::vector<uint32_t>(rec.kp.radix, rec.kp.radix + rec.kp.nf), b.precision, b.dry, twoff);
+    rec.tables.push_back(tw);
+    rec.kp.tw = tw->dptr;
     b.plan->passes.push_back(rec);
     return true;
 }
@@ -2679,6 +2728,18 @@ static void emit_real_step(Builder& b, PassKind kind, uint64_t half, const std::
     b.plan->passes.push_back(rec);
 }
 
+// the axes beside dimension `skip`: the other dimensions and the batch
+static std::vector<Other> other_axes(const View& in, const View& out, const size_t* len, size_t rank,
+                                     size_t batch, size_t skip)
+{
+    std::vector<Other> o;
+    for(size_t d = 0; d < rank; ++d)
+        if(d != skip)
+            o.push_back({(uint32_t)len[d], in.stride[d], out.stride[d]});
+    o.push_back({(uint32_t)batch, in.stride[3], out.stride[3]});
+    return o;
+}
+
 // A single-pass dimension d followed by a long strided dimension e = d+1 (a "column"
 // dimension too long for one column tile, e.g. the second dimension of a 4096 x 4096
 // transform).  The pass over d writes its rows into the work buffer in permuted order (row
@@ -2700,8 +2761,12 @@ static bool emit_dims_staged(Builder& b, const size_t* len, size_t rank, size_t 
     for(size_t i = 0; i < rank; ++i)
         if(i != e && len[i] > 1 && (src.stride[i] < src.stride[e] || out.stride[i] < out.stride[e]))
             column = true;
-    if(!column || !smooth(n) || plain_dim_is_single(n, true, esize, src.stride[e], out.stride[e])
-       || tall_width(n, esize, src.stride[e], out.stride[e]) != 0)
+    if(!column || !smooth(n) || plain_dim_is_single(n, true, esize, src.stride[e], out.stride[e]))
+        return false;
+    // nor one pass of the tall column kernel, which would work in the output array
+    PassRec tall;
+    if(plan_tall(b, n, out.stride[e], out.stride[e], other_axes(out, out, len, rank, batch, e), out.io, out.io, dir, 1.0,
+                 false, tall))
         return false;
     // the tiles of the staged passes are as wide as the rows below dimension e are long; with
     // short rows the plain split is faster (its pass A merges the rows into wider tiles)
@@ -2820,17 +2885,6 @@ static bool emit_dims_staged(Builder& b, const size_t* len, size_t rank, size_t 
 
 // ---------------------------------------------------------------------------
 // whole transforms
-
-static std::vector<Other> other_axes(const View& in, const View& out, const size_t* len, size_t rank,
-                                     size_t batch, size_t skip)
-{
-    std::vector<Other> o;
-    for(size_t d = 0; d < rank; ++d)
-        if(d != skip)
-            o.push_back({(uint32_t)len[d], in.stride[d], out.stride[d]});
-    o.push_back({(uint32_t)batch, in.stride[3], out.stride[3]});
-    return o;
-}
 
 // Even-length real transform whose half length needs a wide kernel: the fused variant, if the
 // layout allows it.  Leaves the pass list untouched and returns false otherwise.

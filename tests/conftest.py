@@ -12,6 +12,14 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu)")
 
 
+@pytest.fixture(autouse=True)
+def small_grids_of_tall_columns(request, monkeypatch):
+    """tests of the tall column kernel run it at sizes too small for it to pay (the edges of its tiles);
+    those of the rule itself say `tall_rule` in their name"""
+    if "tall" in request.node.nodeid and "tall_rule" not in request.node.nodeid:
+        monkeypatch.setenv("ROCFFT_AMD_TALL_ANY_GRID", "1")
+
+
 @pytest.fixture(scope="session")
 def emu():
     """Planner + API linked against the host emulation of the runtime layer."""

@@ -1,11 +1,16 @@
 """Plans with tall column passes (rocfft_amd/csrc/tall_kernels.hip) through the emulation, which runs
 those passes when a test asks for them: what such a plan accepts is what the plan without them does."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
 
+import helpers as H
 import rocfft_amd.binding as B
+from test_callbacks import ROOT, callback_library, check_case
 
 
 @pytest.fixture
@@ -75,3 +80,159 @@ def test_static_area_too_small_for_the_plan_without_tall_columns(tall):
         assert plan.work_buffer_size > B.STATIC_WORK_BYTES
         assert plan.execute_static_status([x.ctypes.data], [y.ctypes.data]) == B.STATUS_INVALID_WORK_BUFFER
         assert (y == 7).all()
+
+
+# (precision, length): both tile widths, idle lanes, four passes, a prime factor of 17
+TALL = [(B.SINGLE, 648), (B.SINGLE, 1020), (B.SINGLE, 1100), (B.SINGLE, 4096), (B.DOUBLE, 750), (B.DOUBLE, 1089),
+        (B.DOUBLE, 2401), (B.DOUBLE, 3528)]
+
+
+@pytest.mark.parametrize("prec,n", TALL, ids=lambda v: str(v))
+def test_parameters_of_tall_columns(tall, prec, n):
+    """The plan's strides, tiles and workgroups, run by a plain transform on exactly those: full tiles,
+    remainders of 1 and W-1 columns, other row pitches, outer dimensions, in place, a scale factor."""
+    before = tall.c.fftrt_emu_tall_launches()
+
+    def columns(kind, cols, pitch=None, out_pitch=None, **kw):
+        p = pitch or cols
+        H.check(tall, H.HostBackend(), kind, [n], cols, prec, in_strides=[p], in_dist=1, out_strides=[out_pitch or p],
+                out_dist=1, **kw)
+
+    columns(B.COMPLEX_FORWARD, 16)
+    columns(B.COMPLEX_INVERSE, 9, scale=0.25)
+    columns(B.COMPLEX_INVERSE, 23, inplace=True)
+    columns(B.COMPLEX_FORWARD, 8, pitch=21, out_pitch=32)
+    columns(B.COMPLEX_FORWARD, 16, in_offsets=[3, 0], out_offsets=[1, 0])
+    H.check(tall, H.HostBackend(), B.COMPLEX_INVERSE, [9, n, 2], 2, prec, inplace=True)
+    H.check(tall, H.HostBackend(), B.REAL_FORWARD, [18, n], 2, prec)
+    H.check(tall, H.HostBackend(), B.REAL_INVERSE, [18, 2, n], 1, prec)
+    assert tall.c.fftrt_emu_tall_launches() - before == 8
+
+
+FORMS = [(B.COMPLEX_FORWARD, B.SINGLE, [24, 1080], 2), (B.COMPLEX_INVERSE, B.DOUBLE, [12, 960], 1),
+         (B.REAL_FORWARD, B.SINGLE, [30, 648], 1), (B.REAL_INVERSE, B.SINGLE, [30, 648], 1),
+         (B.COMPLEX_FORWARD, B.SINGLE, [10000, 648], 1)]
+
+
+@pytest.mark.parametrize("which", ["load", "store", "load+store"])
+def test_callbacks_take_a_list_without_tall_columns_where_they_have_to(tall, which):
+    """A callback on the side of a tall pass sends the call to the other list (behind rows of 10000
+    points to that list's own second list); on the other side the tall pass stays."""
+    cblib = callback_library("libcb_host.so")
+    for kind, prec, lengths, batch in FORMS:
+        assert "tall" in tall.describe(B.NOTINPLACE, kind, prec, lengths, batch)[1], lengths
+        before = tall.c.fftrt_emu_tall_launches()
+        check_case(tall, H.HostBackend(), cblib, kind, lengths, batch, prec, {}, which)
+        at_the_end = kind != B.REAL_INVERSE  # the pass over the columns is the last one, else the first
+        stays = which == ("load" if at_the_end else "store") and lengths[0] < 10000
+        assert tall.c.fftrt_emu_tall_launches() - before == int(stays), (lengths, which)
+
+
+def test_buffers_aligned_to_a_scalar_take_a_list_without_tall_columns(tall):
+    for kind, prec, lengths, batch in FORMS:
+        if kind not in (B.COMPLEX_FORWARD, B.COMPLEX_INVERSE):
+            continue
+        rt = np.float32 if prec == B.SINGLE else np.float64
+        total = 2 * batch * int(np.prod(lengths))
+        x = np.random.default_rng(5).uniform(-1, 1, total).astype(rt)
+        xs, ys = np.zeros(total + 4, dtype=rt), np.zeros(total + 4, dtype=rt)
+        # (numpy's allocations are aligned to 16 bytes)
+        shift = 1
+        xs[shift:shift + total] = x
+        want = np.empty_like(x)
+        plan = B.Plan(B.NOTINPLACE, kind, prec, lengths, batch, lib=tall)
+        before = tall.c.fftrt_emu_tall_launches()
+        plan.execute([x.ctypes.data], [want.ctypes.data])
+        assert tall.c.fftrt_emu_tall_launches() == before + 1
+        plan.execute([xs.ctypes.data + xs.itemsize], [ys.ctypes.data + ys.itemsize])
+        assert tall.c.fftrt_emu_tall_launches() == before + 1
+        scale = np.abs(want).max()
+        assert np.abs(ys[shift:shift + total] - want).max() <= 8 * np.finfo(rt).eps * scale * 4
+        assert ys[0] == 0 and not ys[shift + total:].any()
+
+
+def test_arrays_that_keep_the_passes_they_had(tall):
+    """planar and half-precision arrays, and strides whose offsets inside a tile do not fit 32 bits"""
+    for lengths in ([64, 960], [30, 1080], [128, 4096]):
+        assert "tall" in tall.describe(B.NOTINPLACE, B.COMPLEX_FORWARD, B.SINGLE, lengths, 2)[1]
+        assert "tall" not in tall.describe(B.NOTINPLACE, B.COMPLEX_FORWARD, B.HALF, lengths, 2)[1]
+        for types in ((B.COMPLEX_PLANAR, B.COMPLEX_PLANAR), (B.COMPLEX_PLANAR, B.COMPLEX_INTERLEAVED),
+                      (B.COMPLEX_INTERLEAVED, B.COMPLEX_PLANAR)):
+            desc = B.PlanDescription(lib=tall).set_data_layout(*types)
+            text = tall.describe(B.NOTINPLACE, B.COMPLEX_FORWARD, B.SINGLE, lengths, 2, desc)[1]
+            # (from planar to interleaved the rows write the interleaved array, which the columns then use)
+            assert ("tall" in text) == (types[1] == B.COMPLEX_INTERLEAVED), (lengths, types)
+
+    def columns(pitch):
+        desc = B.PlanDescription(lib=tall)
+        desc.set_data_layout(B.COMPLEX_INTERLEAVED, B.COMPLEX_INTERLEAVED, None, None, [pitch], 1, [pitch], 1)
+        return tall.describe(B.NOTINPLACE, B.COMPLEX_FORWARD, B.SINGLE, [960], 64, desc)[1]
+
+    # (960 + 1) rows of the pitch and a tile of 8 columns stay below 2^32 bytes, or do not
+    last = ((1 << 29) - 8 - 1) // 961
+    assert "tall" in columns(last) and "tall" not in columns(last + 1)
+
+
+def test_switch_without_tall_columns():
+    """the product library's planner (no device needed) with and without ROCFFT_AMD_NO_TALL"""
+    code = ("import rocfft_amd.binding as B; l = B.library();"
+            "print('tall' in l.describe(B.NOTINPLACE, B.COMPLEX_FORWARD, B.SINGLE, [4096, 960], 4)[1])")
+    env = {k: v for k, v in os.environ.items() if not k.startswith("ROCFFT_AMD_")}
+    for extra, want in (({}, "True"), ({"ROCFFT_AMD_NO_TALL": "1"}, "False")):
+        out = subprocess.run([sys.executable, "-c", code], env=dict(env, **extra), cwd=ROOT, capture_output=True,
+                             text=True, timeout=120)
+        assert out.returncode == 0 and out.stdout.split()[-1] == want, (extra, out.stdout, out.stderr[-500:])
+
+
+def is_tall(lib, prec, lengths, batch=1, pitch=None):
+    desc = None
+    if pitch:
+        desc = B.PlanDescription(lib=lib)
+        desc.set_data_layout(B.COMPLEX_INTERLEAVED, B.COMPLEX_INTERLEAVED, None, None, [pitch], 1, [pitch], 1)
+    st, text, _ = lib.describe(B.NOTINPLACE, B.COMPLEX_FORWARD, prec, lengths, batch, desc)
+    assert st == 0
+    return "tall" in text
+
+
+# (precision, points, columns, taken): both sides of each line of tall_pays
+RULE = [
+    # in the place of two passes: more than a quarter of a round of 256 workgroups
+    (B.SINGLE, 960, 512, False), (B.SINGLE, 960, 576, True),
+    # ... three quarters with four radix passes
+    (B.SINGLE, 2025, 1472, False), (B.SINGLE, 2025, 1536, True),
+    # ... four fifths of the last round and those before it
+    (B.SINGLE, 1500, 2560, False), (B.SINGLE, 1500, 3264, False), (B.SINGLE, 1500, 3328, True),
+    # in the place of one pass: seven eighths
+    (B.SINGLE, 880, 1784, False), (B.SINGLE, 880, 1800, True), (B.SINGLE, 880, 3000, False),
+    # 32-byte runs: the same
+    (B.DOUBLE, 3840, 446, False), (B.DOUBLE, 3840, 448, True), (B.DOUBLE, 3840, 768, False),
+    # ... and rows that start on a line where one pass would do
+    (B.DOUBLE, 3000, 1000, True), (B.DOUBLE, 3000, 1001, False),
+    # ... and pitches that are multiples of 512 bytes
+    (B.DOUBLE, 2401, 4096, False), (B.DOUBLE, 2430, 4096, True),
+]
+
+
+@pytest.mark.parametrize("prec,n,cols,taken", RULE, ids=lambda v: str(v))
+def test_tall_rule(tall, prec, n, cols, taken):
+    assert is_tall(tall, prec, [n], cols, cols) == taken
+
+
+def test_tall_rule_counts_idle_columns(tall):
+    """short rows that leave the last tile half empty keep the pass that folds the batch into its tiles"""
+    assert is_tall(tall, B.SINGLE, [15, 1080], 240) and not is_tall(tall, B.SINGLE, [9, 1080], 240)
+    # small problems as a whole: what the tile passes did faster
+    for prec, lengths, batch in ((B.SINGLE, [70, 2048], 1), (B.SINGLE, [10, 1080], 3), (B.DOUBLE, [12, 2048], 1),
+                                 (B.SINGLE, [64, 2187], 1), (B.DOUBLE, [16, 3888], 1)):
+        assert not is_tall(tall, prec, lengths, batch), lengths
+
+
+def test_tall_rule_where_the_pass_is_refused_later(tall):
+    """The rows before a long strided dimension are written in permuted order exactly when that dimension
+    is not one tall pass: here the offsets inside its tiles would not fit 32 bits."""
+    for lengths, want in (([16384, 16, 2000], "tall"), ([16384, 16, 2048], "staged")):
+        st, text, work = tall.describe(B.NOTINPLACE, B.COMPLEX_FORWARD, B.SINGLE, lengths)
+        assert st == 0 and want in text, text
+        tall.c.fftrt_emu_set_tall(0)
+        assert work == tall.describe(B.NOTINPLACE, B.COMPLEX_FORWARD, B.SINGLE, lengths)[2]
+        tall.c.fftrt_emu_set_tall(1)

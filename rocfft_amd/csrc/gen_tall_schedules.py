@@ -21,6 +21,11 @@ COST = {2: 2, 3: 4, 4: 4, 5: 9, 6: 8, 7: 16, 8: 9, 9: 17, 10: 16, 11: 40, 12: 17
 LDS_BYTES = 160 * 1024
 SLICES = 4
 NO_PAD = 31
+# Lengths left out because the passes they would replace are faster: in single precision 714 and 784 points, whose
+# tile pass has 8 columns too (x 4096 columns 18.1 against 20.5 and 20.0 against 23.8 us), 1300 (x 16384 146 against
+# 161 us), 2448 (x 3001 53 against 61 us) and 2601 (x 1500 33 against 38 us); in double 2420 and 2500 with rows of
+# 32 KB and more (1.04x to 1.3x) and 2904 (x 2000 70 against 79 us)
+LEFT_OUT = {False: (714, 784, 1300, 2448, 2601), True: (2420, 2500, 2904)}
 
 
 def pitch(n, shift):
@@ -56,9 +61,9 @@ def exchange_cycles(n, sch, t, width, double, shift):
 
 
 def padding(n, sch, t, width, double):
-    """the padding with the fewest LDS cycles among those that leave the compute unit as many workgroups"""
+    """the padding with the fewest LDS cycles among those whose tiles leave room for as many workgroups"""
     size = width * (16 if double else 8)
-    room = LDS_BYTES // (2 if 2 * pitch(n, 4) * size <= LDS_BYTES and t * width <= 512 else 1)
+    room = LDS_BYTES // (2 if 2 * pitch(n, NO_PAD) * size <= LDS_BYTES and n <= 1200 else 1)
     fit = [s for s in (NO_PAD, 5, 4, 3) if pitch(n, s) * size <= room]
     return min(fit, key=lambda s: (round(exchange_cycles(n, sch, t, width, double, s), 2), -s))
 
@@ -95,20 +100,28 @@ def pick(n, double):
     """schedule, threads per transform and columns per workgroup, or None"""
     if double:
         width = 4 if n <= 2400 else 2
-        # 128 registers a thread: 10 values (and their twiddles), 12 spill a few registers
-        tries = [(n // 12, 1024 // width, 12)] if n <= 1200 else [(n // 10, 1024 // width, 10),
-                                                                 (n // 12, 1024 // width, 12)]
+        tries = [(n // 11, 1024 // width, 11), (n // 12, 1024 // width, 12)]
     else:
         width = 8 if n <= 2400 else 4
-        # up to 1200 points two workgroups share a compute unit; beyond, one: as many threads as it can have
+        # up to 1200 points two workgroups of 512 threads share a compute unit; beyond, one: as many threads as
+        # it can have
         tries = [(64, 128, 18)] if n <= 1200 else [(96, 128, 20)] if n <= 2400 else [(144, 256, 18)] if n <= 3500 else [(200, 256, 17)]
     if pitch(n, 4) * width * (16 if double else 8) > LDS_BYTES:
         return None
+    found = None
     for lo, hi, values in tries:
         b = best(n, lo, hi, values)
-        if b and (double or not 2400 < n <= 3500 or len(b[1]) <= 3):
-            return b[1], b[2], width
-    return None
+        if not b or (not double and 2400 < n <= 3500 and len(b[1]) > 3):
+            continue
+        # Double precision: 11 values of a thread and their twiddles fit 128 registers; 12 take up to 44 bytes
+        # of scratch a lane (76 with two passes of radix 12), which pays where it saves an exchange through LDS
+        # (1200 points x 2048 columns 28.2 against 26.8 us) and not otherwise (750 x 8000 61.9 against 54.2 us).
+        if found and (len(b[1]) >= len(found[1]) or b[1].count(12) > 1):
+            continue
+        if not found and values == 12 and b[1].count(12) > 1:
+            continue
+        found = b
+    return (found[1], found[2], width) if found else None
 
 
 def main():
@@ -123,7 +136,7 @@ def main():
     i = 0
     for n in sorted(x for x in lengths if 640 < x <= 4096):
         for double in (False, True):
-            p = pick(n, double)
+            p = n not in LEFT_OUT[double] and pick(n, double)
             if p:
                 sch = list(p[0]) + [1] * (4 - len(p[0]))
                 print("TALL_SCHED(%d, %s, %d, %d, %d, %d, %d, %d, %d, %d)"

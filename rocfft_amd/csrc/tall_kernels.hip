@@ -7,11 +7,13 @@
 // tile of 64 bytes of neighbouring columns (32 bytes beyond 2400 points, where 160 KB of LDS end).
 // Values go straight from global memory to registers and back; LDS serves the exchanges between
 // the radix passes.  What bounds it is memory: neighbouring tiles complete one another's 128-byte
-// lines in the L2 of one XCD (tile_decode's ranges), and up to 1200 points two workgroups share a
-// compute unit, so that one loads while the other computes.  Single precision, 960 points x 15000
-// columns: 105 -> 55 us (4.2 TB/s); 1080 x 15000 120 -> 68; 2048 x 60000 976 -> 617.  Double, 960 x
-// 25000: 418 -> 219 us; 2400 x 25000 1073 -> 604.  Whole 128-byte tiles (16 columns, one workgroup
-// a compute unit) were slower: 960 x 15000 62 us.
+// lines in the L2 of one XCD (tile_decode's ranges).  Up to 1200 points two workgroups share a compute
+// unit, so that one loads while the other computes, for 129 of 149 kernels; the other 20 have more
+// than 512 threads of more registers than that leaves them, and lose when they are held to those
+// (1190 points x 20000 columns 137 us, held to 80 registers 194 us, the passes before 161 us).  Single precision, arrays that stay in the last-level cache: 960 points x 15000 columns 105 ->
+// 55 us (4.2 TB/s), among other calls 119 -> 79 us; 1080 x 15000 120 -> 68; 2048 x 60000 976 -> 617.
+// Double, 960 x 25000: 418 -> 219 us; 2400 x 25000 1073 -> 604.  Whole 128-byte tiles (16 columns, one
+// workgroup a compute unit) were slower on arrays in that cache: 960 x 15000 62 us.
 #include "fast_core.h"
 #include "tall_registry.h"
 #include "gpu_rt.h"
@@ -68,7 +70,10 @@ struct TallCfg
     static constexpr int PADSHIFT = SHIFT_;
     static constexpr int PITCH    = N_ + ((N_ - 1) >> PADSHIFT); // LDS positions of a column
     static_assert(N_ == R0_ * R1_ * R2_ * R3_, "radices must multiply to N");
-    static_assert(EPT <= 20, "data and twiddles of a thread fit 128 registers");
+    // (data and twiddles of a thread: 20 values in single and 11 in double precision fit 128 registers, 12
+    // in double may take a few of them to scratch memory, see gen_tall_schedules.py)
+    template <typename T>
+    static constexpr bool fits = EPT * sizeof(T) <= 96;
 };
 
 // Where element j of column w lives in LDS: the columns lie beside each other, as in memory, one
@@ -96,6 +101,7 @@ __global__ __launch_bounds__((tall_threads<Cfg, W>()), 4) void tall_kernel(const
     typedef typename cplx_of<T>::type C;
     extern __shared__ double2         tall_smem[];
     C*                                tall_lds = reinterpret_cast<C*>(tall_smem);
+    static_assert(Cfg::template fits<T>, "values of a thread");
     constexpr int            N = Cfg::N, TPT = Cfg::TPT, LAST = Cfg::NP - 1;
     constexpr int            R0 = Cfg::radix(0), S0 = Cfg::S(0), RL = Cfg::radix(LAST), SL = Cfg::S(LAST);
     TileCtx<T>               c;

@@ -2,6 +2,7 @@
 those passes when a test asks for them: what such a plan accepts is what the plan without them does."""
 import ctypes
 import os
+import re
 import subprocess
 import sys
 
@@ -236,3 +237,30 @@ def test_tall_rule_where_the_pass_is_refused_later(tall):
         tall.c.fftrt_emu_set_tall(0)
         assert work == tall.describe(B.NOTINPLACE, B.COMPLEX_FORWARD, B.SINGLE, lengths)[2]
         tall.c.fftrt_emu_set_tall(1)
+
+
+def tall_schedules():
+    """(double precision?, length, radices, threads per transform, columns, padding shift)"""
+    text = open(os.path.join(ROOT, "rocfft_amd", "csrc", "tall_schedules.h")).read()
+    for m in re.finditer(r"^TALL_SCHED\(\d+, (float|double), ([\d, ]+)\)", text, re.M):
+        v = [int(x) for x in m.group(2).split(",")]
+        yield m.group(1) == "double", v[0], [r for r in v[1:5] if r > 1], v[5], v[6], v[7]
+
+
+def test_schedules_fit_registers_and_lds():
+    """At most 12 values of a thread in double precision, one radix-12 pass (two of them took up to 76 bytes
+    of scratch a lane); a padding of the LDS tile never costs the second workgroup of a compute unit."""
+    gen = subprocess.run([sys.executable, os.path.join(ROOT, "rocfft_amd", "csrc", "gen_tall_schedules.py")],
+                         capture_output=True, text=True, check=True).stdout
+    assert gen == open(os.path.join(ROOT, "rocfft_amd", "csrc", "tall_schedules.h")).read()
+    rows = list(tall_schedules())
+    assert len(rows) > 300
+    for double, n, radix, tpt, width, shift in rows:
+        assert int(np.prod(radix)) == n
+        held = max(-(-(n // r) // tpt) * r for r in radix)
+        assert held <= (12 if double else 20) and not (double and radix.count(12) > 1), (n, radix)
+        size = width * (16 if double else 8)
+        lds = (n + ((n - 1) >> shift)) * size
+        assert lds <= 160 * 1024
+        if n <= 1200 and 2 * n * size <= 160 * 1024:
+            assert 2 * lds <= 160 * 1024, (double, n)

@@ -782,7 +782,7 @@ def _plan_text(lib, kind, lengths, batch, prec, cols_pitch=None):
 def test_tall_columns(gpu, prec, n):
     """One pass over long columns: full tiles, a remainder tile of 1 and of W-1 columns, row pitches
     that are line-aligned and that are not, in and out of place, both directions, a scale factor,
-    more outer dimensions, and a buffer aligned to a scalar only (the other pass list)."""
+    more outer dimensions, and arrays that start an odd number of elements into their buffers."""
     lib, be = gpu
     assert "tall column fft" in _plan_text(lib, B.COMPLEX_FORWARD, [n], 32, prec, 32), n
     _columns(lib, be, B.COMPLEX_FORWARD, n, 32, prec)
@@ -799,7 +799,8 @@ def test_tall_columns(gpu, prec, n):
 
 @pytest.mark.parametrize("lengths", [[64, 960], [30, 1080], [128, 4096]])
 def test_tall_columns_in_other_forms(gpu, lengths):
-    """Arrays that kernel does not take keep the passes they had: planar and half precision."""
+    """Arrays that kernel does not take keep the passes they had: planar arrays where the columns lie
+    and half precision."""
     lib, be = gpu
     H.check(lib, be, B.COMPLEX_FORWARD, lengths, 2, B.SINGLE, in_type=B.COMPLEX_PLANAR, out_type=B.COMPLEX_PLANAR)
     H.check(lib, be, B.COMPLEX_FORWARD, lengths, 2, B.DOUBLE, in_type=B.COMPLEX_PLANAR)

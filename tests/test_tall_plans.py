@@ -264,3 +264,13 @@ def test_schedules_fit_registers_and_lds():
         assert lds <= 160 * 1024
         if n <= 1200 and 2 * n * size <= 160 * 1024:
             assert 2 * lds <= 160 * 1024, (double, n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("which", ["load", "store", "load+store"])
+def test_callbacks_beside_tall_columns_on_the_gpu(gpu_lib, which):
+    cblib = callback_library("libcb_device.so")
+    for kind, prec, lengths, batch in FORMS:
+        print("tall callback case", kind, prec, lengths, which, flush=True)
+        assert "tall" in gpu_lib.describe(B.NOTINPLACE, kind, prec, lengths, batch)[1], lengths
+        check_case(gpu_lib, H.TorchBackend(), cblib, kind, lengths, batch, prec, {}, which)

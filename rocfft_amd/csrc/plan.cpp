@@ -2329,43 +2329,56 @@ static uint32_t tall_width(uint64_t n, size_t esize, int64_t is, int64_t os)
 }
 
 // Does one pass of the tall column kernel, `grid` workgroups over rows of `columns` columns, take less
-// time than the passes it would replace?  Measured with all its lengths, 4 to 20000 columns and rows of
-// 5 to 2000 columns in batches (1 to 7500 workgroups), both precisions.
+// time than the passes it would replace?  The lines lie where a sweep of all its lengths over 4 to 20000
+// columns, in and out of place, and over batches of rows of 5 to 2000 columns has the two sides equal
+// (24 500 shapes; 6466 of them are more than 4 % slower with this kernel, up to 1.95x, 13 369 without it).
+// A workgroup transforms twice the columns of a tile pass and many times those of a split, so a grid that
+// leaves most compute units idle costs more than is won in memory, the more the longer the columns are.
 static bool tall_pays(uint64_t n, size_t esize, int64_t is, int64_t os, uint32_t width, uint32_t nf, uint32_t columns,
                       uint64_t grid)
 {
     if(getenv("ROCFFT_AMD_TALL_ANY_GRID")) // (tests of that kernel at small sizes)
         return true;
-    // Idle columns in the last tile of a row, where a tile pass folds the batch into its tile axis:
-    // single precision 880 points, 9 columns x 40 11.9 against 14.7 us, 33 x 16 13.3 against 15.3 us.
-    const uint64_t tiles = ((uint64_t)columns + width - 1) / width;
-    if((uint64_t)columns * 20 < tiles * width * 17)
-        return false;
-    // One workgroup transforms twice the columns of a tile pass and many times those of a split, so a grid
-    // that leaves most compute units idle, or a last round that does, costs more than is won in memory:
-    // 64 columns of 2187 points 9.0 against 15.7 us, 16 of 3888 in double precision 9.3 against 17.7 us.
-    const uint64_t rounds = (grid + 255) / 256;
-    const bool     narrow = width * esize < 64;
-    const bool     one    = plain_dim_is_single(n, true, esize, is, os);
-    const int64_t  line   = 256 / (int64_t)esize; // scalars in 128 bytes
-    if(narrow || one)
+    const bool    dbl     = esize == 16;
+    const int64_t scalar  = (int64_t)esize / 2;
+    const bool    aligned = (is * scalar) % 128 == 0 && (os * scalar) % 128 == 0; // every row starts on a line
+    const bool    pages   = (is * scalar) % 512 == 0 || (os * scalar) % 512 == 0;
+    // idle columns in the last tile of a row count where a tile pass folds the batch into its tile axis
+    const uint64_t slots = ((uint64_t)columns + width - 1) / width * width;
+    if(plain_dim_is_single(n, true, esize, is, os))
     {
-        // In the place of one tile pass, and with 32-byte runs, the gain is 5 to 20 %: all compute units but
-        // for an eighth in every round (3840 points in double precision: 256 columns, half a round, 18.5 against
-        // 22.8 us; 768, one and a half, 43.3 against 48.0 us; but 512, one, 30.8 against 27.9 us with this kernel).
-        // 32-byte runs in the place of one pass need rows that start on a 128-byte line (3000 points x 1000 columns
-        // 64.3 -> 39.0 us, but 2640 x 3001 104 -> 112 us).
-        if(narrow && one && (is % line || os % line))
+        // in the place of one tile pass of the same width: 3 to 40 % faster (single precision 686, 832, 833 and
+        // 896 points: 13 % on many line-aligned rows, but 896 x 256 columns 1.12x, 832 x 5000 in place 1.13x)
+        if(widest_column_tile(n, esize) >= width)
+            return dbl || (n != 686 && n != 832 && n != 833 && n != 896) || (aligned && grid >= 112);
+        // ... of half the width, from where a column's rows fill lines: single precision 880 points x 512 columns
+        // 10.6 -> 10.1 us (x 256 9.1 against 9.8), double 1225 x 384 14.3 -> 11.3 us (x 128 10.1 against 10.3); rows
+        // that start inside lines, 880 x 872 in place 8.5 against 10.3, 1225 x 300 9.3 against 10.4, x 872 21.8 -> 12.6
+        if((uint64_t)columns * 20 < slots * 17)
             return false;
-        return grid * 8 >= rounds * 256 * 7;
+        if(aligned)
+            return grid >= (dbl ? 96 : 64);
+        // (and in single precision the last round of workgroups nearly full: 780 x 2600 in place 13.5 against 16.1)
+        const uint64_t rounds = (grid + 255) / 256;
+        return dbl ? grid >= 144 : grid >= 192 && (rounds == 1 || grid * 20 >= rounds * 256 * 17);
     }
-    // In the place of two passes, single precision: from a quarter of a round on (1080 points x 512 columns the
-    // same 10.5 us either way, x 768 12.8 -> 10.9 us), with four radix passes three quarters (2025 x 1024, half a
-    // round, 20.3 against 23.2 us; x 1536 29.7 -> 25.2 us), and no last round mostly idle (1500 x 2560, one and a
-    // quarter, 33.4 against 36.1 us).
-    if(rounds == 1)
-        return grid >= (nf > 3 ? 192 : 65);
-    return grid * 5 >= rounds * 256 * 4;
+    // in the place of two passes
+    if((uint64_t)columns * 10 < slots * 6)
+        return false;
+    if(width * esize < 64)
+    {
+        // 32-byte runs: 3840 points x 512 columns in double precision 30.5 -> 27.3 us (x 256 18.3 against 23.0), in
+        // single 27.2 -> 26.5 us x 768 (x 512 19.3 against 22.8)
+        if(grid < (!pages ? 80 : !dbl ? 176 : n >= 3400 ? 224 : 96))
+            return false;
+        // (not a round and a bit: 3168 points x 640 columns in place 30.6 against 41.0 us)
+        return !dbl || !aligned || grid <= 256 || grid >= 420;
+    }
+    // double precision 1080 points x 64 columns 8.7 -> 6.5 us, 1600 x 64 9.3 against 11.2; single 750 x 64 7.6 -> 6.7,
+    // 1080 x 768 12.8 -> 11.0 (x 512 the same 10.5), 2025 x 1536 29.8 -> 24.9 (x 1024 20.2 against 23.4)
+    if(dbl)
+        return grid >= (n <= 1300 ? 1 : n <= 1900 ? 33 : 65);
+    return n <= 800 || grid >= (pages && nf > 3 && n > 1800 ? 129 : 65);
 }
 
 // One strided dimension as a pass of the tall column kernel, without its tables; false when the

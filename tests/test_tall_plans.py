@@ -197,19 +197,22 @@ def is_tall(lib, prec, lengths, batch=1, pitch=None):
 
 # (precision, points, columns, taken): both sides of each line of tall_pays
 RULE = [
-    # in the place of two passes: more than a quarter of a round of 256 workgroups
-    (B.SINGLE, 960, 512, False), (B.SINGLE, 960, 576, True),
-    # ... three quarters with four radix passes
-    (B.SINGLE, 2025, 1472, False), (B.SINGLE, 2025, 1536, True),
-    # ... four fifths of the last round and those before it
-    (B.SINGLE, 1500, 2560, False), (B.SINGLE, 1500, 3264, False), (B.SINGLE, 1500, 3328, True),
-    # in the place of one pass: seven eighths
-    (B.SINGLE, 880, 1784, False), (B.SINGLE, 880, 1800, True), (B.SINGLE, 880, 3000, False),
-    # 32-byte runs: the same
-    (B.DOUBLE, 3840, 446, False), (B.DOUBLE, 3840, 448, True), (B.DOUBLE, 3840, 768, False),
-    # ... and rows that start on a line where one pass would do
-    (B.DOUBLE, 3000, 1000, True), (B.DOUBLE, 3000, 1001, False),
-    # ... and pitches that are multiples of 512 bytes
+    # in the place of one pass of the same width: always; four lengths from 112 workgroups on full lines
+    (B.SINGLE, 704, 8, True), (B.DOUBLE, 1200, 5, True), (B.DOUBLE, 3000, 17, True),
+    (B.SINGLE, 896, 880, False), (B.SINGLE, 896, 912, True), (B.SINGLE, 896, 913, False),
+    # ... of half the width, rows that start on lines and rows that do not
+    (B.SINGLE, 880, 496, False), (B.SINGLE, 880, 528, True), (B.SINGLE, 880, 1521, False), (B.SINGLE, 880, 1530, True),
+    (B.SINGLE, 880, 2600, False), (B.SINGLE, 880, 3601, True),
+    (B.DOUBLE, 1225, 376, False), (B.DOUBLE, 1225, 392, True), (B.DOUBLE, 1225, 570, False), (B.DOUBLE, 1225, 573, True),
+    # in the place of two passes
+    (B.SINGLE, 750, 8, True), (B.SINGLE, 960, 512, False), (B.SINGLE, 960, 576, True),
+    (B.SINGLE, 2025, 1024, False), (B.SINGLE, 2025, 1088, True), (B.SINGLE, 2048, 512, False), (B.SINGLE, 2048, 576, True),
+    (B.DOUBLE, 1080, 32, True), (B.DOUBLE, 1600, 128, False), (B.DOUBLE, 1600, 160, True),
+    (B.DOUBLE, 2187, 256, False), (B.DOUBLE, 2187, 288, True),
+    # ... with 32-byte runs, among them pitches that are multiples of 512 bytes
+    (B.SINGLE, 3840, 640, False), (B.SINGLE, 3840, 704, True), (B.SINGLE, 3840, 315, False), (B.SINGLE, 3840, 321, True),
+    (B.DOUBLE, 2816, 160, False), (B.DOUBLE, 2816, 192, True), (B.DOUBLE, 3840, 416, False), (B.DOUBLE, 3840, 448, True),
+    (B.DOUBLE, 3168, 640, False), (B.DOUBLE, 3168, 864, True),
     (B.DOUBLE, 2401, 4096, False), (B.DOUBLE, 2430, 4096, True),
 ]
 
@@ -222,9 +225,10 @@ def test_tall_rule(tall, prec, n, cols, taken):
 def test_tall_rule_counts_idle_columns(tall):
     """short rows that leave the last tile half empty keep the pass that folds the batch into its tiles"""
     assert is_tall(tall, B.SINGLE, [15, 1080], 240) and not is_tall(tall, B.SINGLE, [9, 1080], 240)
+    assert is_tall(tall, B.SINGLE, [15, 880], 240) and not is_tall(tall, B.SINGLE, [13, 880], 240)
     # small problems as a whole: what the tile passes did faster
-    for prec, lengths, batch in ((B.SINGLE, [70, 2048], 1), (B.SINGLE, [10, 1080], 3), (B.DOUBLE, [12, 2048], 1),
-                                 (B.SINGLE, [64, 2187], 1), (B.DOUBLE, [16, 3888], 1)):
+    for prec, lengths, batch in ((B.SINGLE, [70, 2048], 1), (B.SINGLE, [10, 1080], 3), (B.DOUBLE, [12, 2160], 1),
+                                 (B.SINGLE, [64, 2187], 1), (B.DOUBLE, [16, 3993], 1)):
         assert not is_tall(tall, prec, lengths, batch), lengths
 
 

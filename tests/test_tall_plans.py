@@ -107,7 +107,10 @@ def test_parameters_of_tall_columns(tall, prec, n):
     H.check(tall, H.HostBackend(), B.COMPLEX_INVERSE, [9, n, 2], 2, prec, inplace=True)
     H.check(tall, H.HostBackend(), B.REAL_FORWARD, [18, n], 2, prec)
     H.check(tall, H.HostBackend(), B.REAL_INVERSE, [18, 2, n], 1, prec)
-    assert tall.c.fftrt_emu_tall_launches() - before == 8
+    # rows as long as the permuted staging of a split wants them, another pitch on the input side
+    H.check(tall, H.HostBackend(), B.COMPLEX_FORWARD, [72, n], 1, prec, in_strides=[1, 512], in_dist=512 * n,
+            out_strides=[1, 80], out_dist=80 * n)
+    assert tall.c.fftrt_emu_tall_launches() - before == 9
 
 
 FORMS = [(B.COMPLEX_FORWARD, B.SINGLE, [24, 1080], 2), (B.COMPLEX_INVERSE, B.DOUBLE, [12, 960], 1),

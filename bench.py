@@ -470,12 +470,15 @@ def copy_probes():
         "tiles 4096 x 1 (contiguous rows of 32 KiB), one workgroup per tile": dict(tiles, tile_width=256, in_row=256, out_row=256, tiles_per_slab=1, rows=32768, in_slab=4096, out_slab=4096),
         "tiles 4096 x 1, nontemporal": dict(tiles, tile_width=256, in_row=256, out_row=256, tiles_per_slab=1, rows=32768, in_slab=4096, out_slab=4096, nontemporal=1),
         "tiles 4096 x 1, resident grid": dict(tiles, tile_width=256, in_row=256, out_row=256, tiles_per_slab=1, rows=32768, in_slab=4096, out_slab=4096, resident_grid=1),
-        # configuration 3, column passes over 8 arrays of 4096 rows of 4096 elements: a tile is 64
-        # columns x 64 rows, the rows adjacent (first pass of the split) or 64 rows apart (second pass)
-        "tiles 64 x 64, adjacent rows of 4096 (configuration 3, first column pass)": dict(tiles, in_row=4096, out_row=4096, tiles_per_slab=64, rows=512, in_slab=64 * 4096, out_slab=64 * 4096),
+        # configuration 3, the column pass over 8 arrays of 4096 rows of 4096 elements: a tile is 4 whole columns
+        "tiles 4 x 4096, rows of 4096, each XCD a range of tiles (configuration 3, columns)": dict(shape=B.PROBE_TALL_TILES, tile_width=4, elem_bytes=8, in_row=4096, out_row=4096, tiles_per_slab=1024, rows=8, in_slab=4096 * 4096, out_slab=4096 * 4096, xcd_ranges=1),
+        "tiles 4 x 4096, rows 4096 + 16 apart, each XCD a range of tiles": dict(shape=B.PROBE_TALL_TILES, tile_width=4, elem_bytes=8, in_row=4112, out_row=4112, tiles_per_slab=1024, rows=8, in_slab=4112 * 4096, out_slab=4112 * 4096, xcd_ranges=1),
+        # the same arrays in the two column passes of a split (planar arrays, other pitches): a tile is 64
+        # columns x 64 rows, the rows adjacent (first pass) or 64 rows apart (second pass)
+        "tiles 64 x 64, adjacent rows of 4096 (first column pass of a split)": dict(tiles, in_row=4096, out_row=4096, tiles_per_slab=64, rows=512, in_slab=64 * 4096, out_slab=64 * 4096),
         "tiles 64 x 64, adjacent rows of 4096, nontemporal": dict(tiles, in_row=4096, out_row=4096, tiles_per_slab=64, rows=512, in_slab=64 * 4096, out_slab=64 * 4096, nontemporal=1),
         "tiles 64 x 64, adjacent rows of 4096, resident grid": dict(tiles, in_row=4096, out_row=4096, tiles_per_slab=64, rows=512, in_slab=64 * 4096, out_slab=64 * 4096, resident_grid=1),
-        "tiles 64 x 64, rows 64 x 4096 apart (configuration 3, second column pass)": dict(tiles, in_row=64 * 4096, out_row=64 * 4096, tiles_per_slab=64, rows=512, in_slab=4096, out_slab=4096, slabs_inner=64, in_slab_outer=4096 * 4096, out_slab_outer=4096 * 4096),
+        "tiles 64 x 64, rows 64 x 4096 apart (second column pass of a split)": dict(tiles, in_row=64 * 4096, out_row=64 * 4096, tiles_per_slab=64, rows=512, in_slab=4096, out_slab=4096, slabs_inner=64, in_slab_outer=4096 * 4096, out_slab_outer=4096 * 4096),
         "tiles 64 x 64, rows 64 x 4096 apart, nontemporal": dict(tiles, in_row=64 * 4096, out_row=64 * 4096, tiles_per_slab=64, rows=512, in_slab=4096, out_slab=4096, slabs_inner=64, in_slab_outer=4096 * 4096, out_slab_outer=4096 * 4096, nontemporal=1),
         "tiles 64 x 64, adjacent rows 4096 + 32 apart (256 bytes of padding)": dict(tiles, in_row=4128, out_row=4128, tiles_per_slab=64, rows=512, in_slab=64 * 4128, out_slab=64 * 4128),
         "tiles 64 x 64, adjacent rows 4096 + 64 apart (512 bytes of padding)": dict(tiles, in_row=4160, out_row=4160, tiles_per_slab=64, rows=512, in_slab=64 * 4160, out_slab=64 * 4160),
@@ -505,6 +508,8 @@ def copy_ceilings(torch, lib, names=None, reps=10):
             moved = 2.0 * f["rows"] * 32768 * 8
         elif f["shape"] == B.PROBE_TILES:
             moved = 2.0 * f["tiles_per_slab"] * f["rows"] * 4096 * f["elem_bytes"]
+        elif f["shape"] == B.PROBE_TALL_TILES:
+            moved = 2.0 * f["tiles_per_slab"] * f["rows"] * 16384 * f["elem_bytes"]
         elif f["shape"] == B.PROBE_STREAM:
             moved = 2.0 * f["bytes"]
         else:
@@ -532,7 +537,7 @@ def copy_ceilings(torch, lib, names=None, reps=10):
 SHAPE_OF_CONFIG = {
     1: "tiles 4096 x 1 (contiguous rows of 32 KiB), one workgroup per tile",
     2: "rows 32769 apart read, rows of 32768 written (real inverse), 32/32",
-    3: "tiles 64 x 64, rows 64 x 4096 apart (configuration 3, second column pass)",
+    3: "tiles 4 x 4096, rows of 4096, each XCD a range of tiles (configuration 3, columns)",
     4: "tiles 8 x 512 of 16 B, rows 131584 apart (configuration 4, z columns)",
     5: "tiles 4096 x 1 (contiguous rows of 32 KiB), one workgroup per tile",
 }

@@ -98,10 +98,12 @@ enum rocfft_amd_probe_shape
     ROCFFT_AMD_PROBE_ROWS   = 3, /* `rows` rows of 32768 elements of 8 bytes, one workgroup of 1024 threads per
                                     row, `group` (8 or 32) loads then as many stores at a time; rows in_row /
                                     out_row elements apart */
-    ROCFFT_AMD_PROBE_TILES  = 4  /* tiles of tile_width x (4096 / tile_width) elements of elem_bytes (8 or 16),
+    ROCFFT_AMD_PROBE_TILES  = 4, /* tiles of tile_width x (4096 / tile_width) elements of elem_bytes (8 or 16),
                                     one workgroup of 256 threads per tile, 16 loads then 16 stores per thread;
                                     tile rows in_row / out_row elements apart; tiles_per_slab tiles side by
                                     side, `rows` slabs in_slab / out_slab elements apart */
+    ROCFFT_AMD_PROBE_TALL_TILES = 5 /* the same with 1024 threads and tiles of tile_width x (16384 / tile_width)
+                                       elements: the shape of the tall column passes */
 };
 typedef struct rocfft_amd_probe
 {

@@ -107,7 +107,7 @@ class Probe(ctypes.Structure):
                 ("slabs_inner", ctypes.c_uint), ("in_slab_outer", ctypes.c_size_t), ("out_slab_outer", ctypes.c_size_t)]
 
 
-PROBE_STREAM, PROBE_READ, PROBE_WRITE, PROBE_ROWS, PROBE_TILES = range(5)
+PROBE_STREAM, PROBE_READ, PROBE_WRITE, PROBE_ROWS, PROBE_TILES, PROBE_TALL_TILES = range(6)
 
 # size of the device-resident work area behind rocfft_amd_execute_static
 STATIC_WORK_BYTES = 64 << 20

@@ -82,19 +82,19 @@ __global__ __launch_bounds__(1024) void probe_rows(const v2f* in, v2f* out, size
     }
 }
 
-// A tile pass's shape: a workgroup of 256 threads moves a tile of W x (4096 / W) elements
-// (W neighbouring elements are contiguous, the rows of the tile are in_row / out_row elements
+// A tile pass's shape: a workgroup of THREADS threads (256 for the tile passes, 1024 for the tall column
+// passes) moves a tile of W x (16 THREADS / W) elements (W neighbouring elements are contiguous, the rows of the tile are in_row / out_row elements
 // apart), 16 elements per thread, all loads and then all stores; tiles are numbered along the
 // contiguous axis first (tiles_per_slab of them), then by slab (in_slab / out_slab elements apart;
 // with slabs_inner set, in two levels: slabs_inner slabs that far apart, groups of them
 // in_outer / out_outer apart).
-template <typename V>
-__global__ __launch_bounds__(256) void probe_tiles(const V* in, V* out, uint32_t W, size_t in_row, size_t out_row,
+template <typename V, int THREADS>
+__global__ __launch_bounds__(THREADS) void probe_tiles(const V* in, V* out, uint32_t W, size_t in_row, size_t out_row,
                                                    uint32_t tiles_per_slab, size_t in_slab, size_t out_slab,
                                                    uint32_t total, int nt, int xcd_ranges, uint32_t slabs_inner,
                                                    size_t in_outer, size_t out_outer)
 {
-    const uint32_t w = threadIdx.x % W, q = threadIdx.x / W, step = 256 / W;
+    const uint32_t w = threadIdx.x % W, q = threadIdx.x / W, step = (uint32_t)THREADS / W;
     for(uint32_t b0 = blockIdx.x; b0 < total; b0 += gridDim.x)
     {
         uint32_t b = b0;
@@ -191,6 +191,7 @@ extern "C" int fftrt_copy_probe(const struct rocfft_amd_probe* q, void* stream)
         break;
     }
     case ROCFFT_AMD_PROBE_TILES:
+    case ROCFFT_AMD_PROBE_TALL_TILES:
     {
         const uint32_t W = q->tile_width;
         if(!q->src || W == 0 || W > 256 || (W & (W - 1)) || q->rows == 0 || q->tiles_per_slab == 0)
@@ -200,18 +201,24 @@ extern "C" int fftrt_copy_probe(const struct rocfft_amd_probe* q, void* stream)
             return (int)hipErrorInvalidValue;
         const uint32_t grid = (uint32_t)std::min<uint64_t>(total, q->resident_grid ? (uint64_t)per_cu * cus : total);
         const int      xcd  = (q->xcd_ranges && grid == total) ? 1 : 0;
-        if(q->elem_bytes == 8)
-            hipLaunchKernelGGL(probe_tiles<v2f>, dim3(grid), dim3(256), 0, s, static_cast<const v2f*>(q->src),
-                               static_cast<v2f*>(q->dst), W, q->in_row, q->out_row, q->tiles_per_slab, q->in_slab,
-                               q->out_slab, (uint32_t)total, q->nontemporal, xcd, q->slabs_inner, q->in_slab_outer,
-                               q->out_slab_outer);
-        else if(q->elem_bytes == 16)
-            hipLaunchKernelGGL(probe_tiles<v4f>, dim3(grid), dim3(256), 0, s, static_cast<const v4f*>(q->src),
-                               static_cast<v4f*>(q->dst), W, q->in_row, q->out_row, q->tiles_per_slab, q->in_slab,
-                               q->out_slab, (uint32_t)total, q->nontemporal, xcd, q->slabs_inner, q->in_slab_outer,
-                               q->out_slab_outer);
-        else
+        if(q->elem_bytes != 8 && q->elem_bytes != 16)
             return (int)hipErrorInvalidValue;
+#define PROBE_TILES(V, THREADS)                                                                                        \
+    hipLaunchKernelGGL((probe_tiles<V, THREADS>), dim3(grid), dim3(THREADS), 0, s, static_cast<const V*>(q->src),      \
+                       static_cast<V*>(q->dst), W, q->in_row, q->out_row, q->tiles_per_slab, q->in_slab, q->out_slab,  \
+                       (uint32_t)total, q->nontemporal, xcd, q->slabs_inner, q->in_slab_outer, q->out_slab_outer)
+        if(q->shape == ROCFFT_AMD_PROBE_TILES)
+        {
+            if(q->elem_bytes == 8)
+                PROBE_TILES(v2f, 256);
+            else
+                PROBE_TILES(v4f, 256);
+        }
+        else if(q->elem_bytes == 8)
+            PROBE_TILES(v2f, 1024);
+        else
+            PROBE_TILES(v4f, 1024);
+#undef PROBE_TILES
         break;
     }
     default:

@@ -79,6 +79,18 @@ def test_probe_shapes_copy_what_they_claim(gpu_lib):
     m = 2 * 4 * 16 * 512 * 4  # two groups of 512 x 4 rows of 16 elements of four floats
     assert torch.equal(dst[:m], src[:m]) and (dst[m:] == -1).all()
 
+    # the tall tiles: 4 x 4096 elements of 8 bytes, 16 side by side in two slabs; 8 x 2048 of 16 bytes
+    for extra in ({}, {"xcd_ranges": 1}):
+        for width, elem, row, per_slab in ((4, 8, 64, 16), (8, 16, 16, 2)):
+            dst = fresh()
+            slab = row * (16384 // width)
+            lib.copy_probe(stream, shape=B.PROBE_TALL_TILES, src=src.data_ptr(), dst=dst.data_ptr(), tile_width=width,
+                           elem_bytes=elem, in_row=row, out_row=row, tiles_per_slab=per_slab, rows=2, in_slab=slab,
+                           out_slab=slab, **extra)
+            torch.cuda.synchronize()
+            m = 2 * slab * elem // 4
+            assert m < n and torch.equal(dst[:m], src[:m]) and (dst[m:] == -1).all(), (width, extra)
+
     # refused: a byte count that is no multiple of 16, no destination, rows shorter than 32768
     for bad in (dict(shape=B.PROBE_STREAM, src=src.data_ptr(), dst=dst.data_ptr(), bytes=100),
                 dict(shape=B.PROBE_STREAM, src=src.data_ptr(), dst=0, bytes=1024),

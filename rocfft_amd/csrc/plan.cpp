@@ -2303,14 +2303,16 @@ static uint32_t tall_width(uint64_t n, size_t esize, int64_t is, int64_t os)
     // Single precision, rows that do not start on a 128-byte line: a tile pass of 4 columns whose
     // LDS lets three workgroups share a compute unit beats one workgroup of this kernel (1536 points
     // x 50001 columns 425 against 478 us; with line-aligned rows 139 against 95 us for x 12000).
-    // Where two workgroups of this kernel fit (up to 1200 points) it wins either way.
+    // Where the LDS has room for two workgroups of this kernel (up to 1200 points) it is as fast or faster
+    // either way (1190 x 3001 33.2 -> 31.2 us).
     const int64_t line = 256 / (int64_t)esize; // scalars
     const size_t  col  = (size_t)lds_pitch((uint32_t)n) * esize;
     if(esize == 8 && (is % line || os % line) && now >= 4 && 3 * 4 * col <= LDS_HARD_BYTES && 2 * 8 * col > LDS_HARD_BYTES)
         return 0;
     if(!fftrt_tall_info(esize == 16 ? 1 : 0, (uint32_t)n, radix, &nf, &tpt, &width, &threads, &pitch))
         return 0;
-    // 32-byte runs at multiples of 512 bytes alias onto few HBM channels.  Single precision, against
+    // 32-byte runs at multiples of 512 bytes alias onto few HBM channels (the lines below lie on the safe
+    // side: at many of the pitches they exclude this kernel takes 0.7 to 0.97 of the time).  Single precision, against
     // the staged split: rows of 32 KB 4096 x 4096 x 8 1153 -> 1135 us and x 1 144 -> 119 us, rows of 24 KB
     // 3072 x 3840 x 3 364 -> 343 us, but rows of 64 KB 8192 x 4096 x 2 620 -> 667 us; up to 3500 points
     // also closer rows lose (15 KB, 1920 x 3072 x 4: 238 -> 247 us).  Double precision: rows of 48 KB
@@ -2754,8 +2756,8 @@ static std::vector<Other> other_axes(const View& in, const View& out, const size
 }
 
 // A single-pass dimension d followed by a long strided dimension e = d+1 (a "column"
-// dimension too long for one column tile, e.g. the second dimension of a 4096 x 4096
-// transform).  The pass over d writes its rows into the work buffer in permuted order (row
+// dimension too long for one column tile and not one tall column pass either, e.g. the second
+// dimension of an 8192 x 4096 transform).  The pass over d writes its rows into the work buffer in permuted order (row
 // n1*n0 + n0' of dimension e goes to slot n0'*n1 + n1): pass A of the split then reads n1
 // consecutive rows where the plain split reads rows n0 apart, and pass B reads the strided rows
 // before writing the user's output.  Measured on MI355X against the plain split of the same

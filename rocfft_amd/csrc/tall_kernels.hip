@@ -10,10 +10,13 @@
 // lines in the L2 of one XCD (tile_decode's ranges).  Up to 1200 points two workgroups share a compute
 // unit, so that one loads while the other computes, for 129 of 149 kernels; the other 20 have more
 // than 512 threads of more registers than that leaves them, and lose when they are held to those
-// (1190 points x 20000 columns 137 us, held to 80 registers 194 us, the passes before 161 us).  Single precision, arrays that stay in the last-level cache: 960 points x 15000 columns 105 ->
-// 55 us (4.2 TB/s), among other calls 119 -> 79 us; 1080 x 15000 120 -> 68; 2048 x 60000 976 -> 617.
-// Double, 960 x 25000: 418 -> 219 us; 2400 x 25000 1073 -> 604.  Whole 128-byte tiles (16 columns, one
-// workgroup a compute unit) were slower on arrays in that cache: 960 x 15000 62 us.
+// (1190 points x 20000 columns 137 us, held to 80 registers 194 us, the passes before 161 us).
+// Single precision, arrays that stay in the last-level cache: 960 points x 15000 columns 105 -> 55 us
+// (4.2 TB/s), among other calls 119 -> 77 us; 1080 x 15000 120 -> 68; 2048 x 60000 976 -> 617.  Double,
+// 960 x 25000: 418 -> 219 us; 2400 x 25000 1073 -> 604.  Whole 128-byte tiles (16 columns, one workgroup
+// a compute unit) were slower on arrays in that cache: 960 x 15000 62 us.  Lines are read and written
+// once (1 to 4 % more than needed) with 64-byte runs; with 32-byte runs 26 % more are written, and
+// 4096 x 4096 x 8 takes 0.735 ms, a plain copy of its shape 0.737 ms.
 #include "fast_core.h"
 #include "tall_registry.h"
 #include "gpu_rt.h"
